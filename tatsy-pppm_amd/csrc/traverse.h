@@ -74,11 +74,17 @@ struct QuadRay {
     RayPre pre;  // pre.o is the origin
     float ix, iy, iz, ox, oy, oz;
     float tmin, t;  // t: the closest hit so far
-    float t_far;    // t * SLAB_FAR_SCALE
+    float t_far;    // slab_limit(t)
     int32_t cur;    // the next inner node (>= 0), a leaf root (< 0), or EMPTY_REF: no ray
     int32_t sp;     // bytes of the stack in use; the lowest entry is EMPTY_REF
     int32_t slot;   // whose ray it is
 };
+
+// What a box's entry distance is held against for a closest hit at t: never
+// infinite, so that an empty slot, entered at infinity, is missed also by a ray
+// without a limit (t infinite, so near the largest float that scaling it
+// overflows, or NaN).
+__device__ inline float slab_limit(float t) { return fminf(t * SLAB_FAR_SCALE, 3.402823466e+38f); }
 
 // The wave's waiting rays: ring positions [head, tail), the same in every lane.
 struct RayQueue {
@@ -163,7 +169,7 @@ __device__ inline void rays_trace(const SceneDev& sc, const WaveRays& w, QuadRay
                 q.oz = a.z * b.z;
                 q.tmin = e.x;
                 q.t = e.y;
-                q.t_far = e.y * SLAB_FAR_SCALE;
+                q.t_far = slab_limit(e.y);
                 q.cur = sc.root;
                 q.sp = STACK_STEP;
                 wave_lds_fence();
@@ -258,7 +264,7 @@ __device__ inline void rays_trace(const SceneDev& sc, const WaveRays& w, QuadRay
             const uint32_t won = (uint32_t)(__ballot(wins) >> (lane & ~3)) & 3u;
             if (won != 0u) {
                 q.t = won & 2u ? __int_as_float(quad_read<QUAD_LANE1>(__float_as_int(h.t))) : t0;
-                q.t_far = q.t * SLAB_FAR_SCALE;
+                q.t_far = slab_limit(q.t);
                 if (c == (int)(won >> 1)) w.slot[q.slot] = make_float4(h.t, __int_as_float(tri), h.u, h.v);
             }
             leaf = q.cur;
