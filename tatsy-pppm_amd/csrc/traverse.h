@@ -207,13 +207,21 @@ __device__ inline void rays_trace(const SceneDev& sc, const WaveRays& w, QuadRay
                 const int at = (int)(((uint32_t)q.cur << 7) | ((uint32_t)c << 5));
                 const v4u p = __builtin_amdgcn_raw_buffer_load_b128(nbuf, at, 0, 0);
                 const v4u r = __builtin_amdgcn_raw_buffer_load_b128(nbuf, at, 16, 0);
-                const float x0 = __uint_as_float(p.x) * q.ix - q.ox, x1 = __uint_as_float(p.w) * q.ix - q.ox;
-                const float y0 = __uint_as_float(p.y) * q.iy - q.oy, y1 = __uint_as_float(r.x) * q.iy - q.oy;
-                const float z0 = __uint_as_float(p.z) * q.iz - q.oz, z1 = __uint_as_float(r.y) * q.iz - q.oz;
-                const float n = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)),
-                                      fmaxf(fminf(z0, z1), ZERO_TMIN ? 0.0f : q.tmin));
-                const float f = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1));
-                const bool hit = n <= f * SLAB_FAR_SCALE && n <= q.t_far;
+                // the near and the far plane of each axis by the direction's sign: an
+                // axis whose products are infinities of both signs (a direction
+                // component whose reciprocal overflows) has a NaN for a plane,
+                // which must not limit the interval, while min and max of the two
+                // planes would take the other one for both
+                const bool fx = q.ix >= 0.0f, fy = q.iy >= 0.0f, fz = q.iz >= 0.0f;
+                const float x0 = __uint_as_float(fx ? p.x : p.w) * q.ix - q.ox;
+                const float x1 = __uint_as_float(fx ? p.w : p.x) * q.ix - q.ox;
+                const float y0 = __uint_as_float(fy ? p.y : r.x) * q.iy - q.oy;
+                const float y1 = __uint_as_float(fy ? r.x : p.y) * q.iy - q.oy;
+                const float z0 = __uint_as_float(fz ? p.z : r.y) * q.iz - q.oz;
+                const float z1 = __uint_as_float(fz ? r.y : p.z) * q.iz - q.oz;
+                const float n = fmaxf(fmaxf(x0, y0), fmaxf(z0, ZERO_TMIN ? 0.0f : q.tmin));
+                const float f = fminf(fminf(x1, y1), z1);
+                const bool hit = n <= fminf(f * SLAB_FAR_SCALE, q.t_far);
                 // the children hit go on the stack farthest first, the nearest
                 // on top, which is taken next; the missed ones above it, where
                 // they do not count.  So lane c writes its child at the number

@@ -3,10 +3,14 @@
 tmax may be infinite, FLT_MAX or NaN (no limit): such a ray meets what one with a limit far
 beyond the scene meets, bit for bit.  The scenes leave nodes with fewer than
 four children, whose empty slots are what a limit without a bound could meet.
+
+A component of the direction may be so small that its reciprocal overflows:
+the ray meets what the oracle's test of every triangle finds.
 """
 import numpy as np
 import pytest
 
+import oracle as O
 import pppm_amd as P
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +67,27 @@ def test_a_limit_without_a_bound(gpu_ctx, kind, builder):
         assert np.array_equal(got["tri"], want["tri"])
         assert np.array_equal(got[hit].view(np.uint32), want[hit].view(np.uint32))
         assert np.array_equal(got["t"][~hit], r["tmax"][~hit], equal_nan=True)
+
+
+@pytest.mark.parametrize("tiny", [1e-40, -1e-40, 1.5e-45])
+@pytest.mark.parametrize("kind", [3, 5, 17, "box"])
+def test_directions_whose_reciprocal_overflows(gpu_ctx, kind, tiny):
+    print(f"[case] scene {kind}, components of {tiny}", flush=True)
+    s = _scene(kind)
+    rays = _rays(np.asarray(s.tri), 6000, 11)
+    # about the origin: planes and rays on both sides of zero, whose products
+    # with an infinite reciprocal are infinities of both signs
+    off = np.float32(2.5)
+    tri = (np.asarray(s.tri).reshape(-1, 3) - off).reshape(np.asarray(s.tri).shape)
+    s = P.Scene(tri, s.bsdf_id, s.bsdfs, s.lights, s.camera, [v - 2.5 for v in s.bbox_min],
+                [v - 2.5 for v in s.bbox_max])
+    rays["origin"] -= off
+    d = rays["dir"].copy()
+    d[d == 0.0] = np.float32(tiny)
+    rays["dir"] = d
+    gpu_ctx.upload(s)
+    gpu_ctx.build_bvh()
+    got = gpu_ctx.intersect(rays)["tri"]
+    _, ref = O.OracleScene(s).intersect(rays.view(np.float32).reshape(-1, 8), brute=True)
+    # a few rays run within a face of a box or along an edge of two triangles
+    assert (ref >= 0).sum() > 1000 and (got != ref).sum() <= 0.002 * len(rays)
