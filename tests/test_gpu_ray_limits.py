@@ -67,6 +67,13 @@ def test_a_limit_without_a_bound(gpu_ctx, kind, builder):
         assert np.array_equal(got["tri"], want["tri"])
         assert np.array_equal(got[hit].view(np.uint32), want[hit].view(np.uint32))
         assert np.array_equal(got["t"][~hit], r["tmax"][~hit], equal_nan=True)
+    # the other end: what lies behind the origin counts too
+    rays["tmin"] = -1e30
+    want = gpu_ctx.intersect(rays)
+    for tmin in (-FLT_MAX, np.float32(-np.inf), np.float32(np.nan)):
+        r = rays.copy()
+        r["tmin"] = tmin
+        assert np.array_equal(gpu_ctx.intersect(r).view(np.uint32), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("tiny", [1e-40, -1e-40, 1.5e-45])
