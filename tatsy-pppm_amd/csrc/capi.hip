@@ -123,36 +123,6 @@ uint32_t* origin_order(Ctx* c, hipStream_t s, int64_t slots, int64_t n, const Gr
     return c->u[4].as<uint32_t>();
 }
 
-// Device memory to the caller's (pageable) memory, complete on return, through
-// two pinned buffers of the context, one copied out while the other fills: the
-// runtime's own way pins the caller's pages, which costs more at every size
-// (32 KB 28 -> 18 us, 0.4 MB 194 -> 48, 6 MB 0.50 -> 0.36 ms, 54 MB 5.3 -> 4.3 ms).
-#define STAGE_BYTES ((size_t)1 << 20)
-hipError_t copy_to_host(Ctx* c, hipStream_t s, void* dst, const void* src, size_t bytes) {
-    hipError_t e;
-    if (!c->stage) {
-        if ((e = hipHostMalloc((void**)&c->stage, 2 * STAGE_BYTES, hipHostMallocDefault)) != hipSuccess) return e;
-        for (auto& ev : c->stage_ev)
-            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
-    }
-    const size_t chunks = (bytes + STAGE_BYTES - 1) / STAGE_BYTES;
-    for (size_t k = 0; k <= chunks; k++) {
-        if (k < chunks) {
-            const size_t at = k * STAGE_BYTES;
-            if ((e = hipMemcpyAsync(c->stage + (k & 1) * STAGE_BYTES, (const char*)src + at,
-                                    std::min(STAGE_BYTES, bytes - at), hipMemcpyDeviceToHost, s)) != hipSuccess)
-                return e;
-            if ((e = hipEventRecord(c->stage_ev[k & 1], s)) != hipSuccess) return e;
-        }
-        if (k > 0) {
-            const size_t at = (k - 1) * STAGE_BYTES;
-            if ((e = hipEventSynchronize(c->stage_ev[(k - 1) & 1])) != hipSuccess) return e;
-            std::memcpy((char*)dst + at, c->stage + ((k - 1) & 1) * STAGE_BYTES, std::min(STAGE_BYTES, bytes - at));
-        }
-    }
-    return hipSuccess;
-}
-
 hipError_t ensure_sort_buffers(Ctx* c, int64_t n, uint32_t S) {
     for (int i = 0; i < 5; i++) {
         hipError_t e = c->u[i].ensure(sizeof(uint32_t) * (size_t)(n > 0 ? n : 1));
@@ -425,7 +395,7 @@ int pppm_intersect(void* ctx_raw, const pppm_ray* rays, int64_t n, pppm_hit* hit
     TRY_HIP(ctx, hipMemcpyAsync(dr, rays, sizeof(pppm_ray) * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
     launch_intersect(ctx->stream, ctx->scene_dev(), dr, n, dh, ctx->cu);
     TRY_HIP(ctx, hipGetLastError());
-    TRY_HIP(ctx, copy_to_host(ctx, ctx->stream, hits, dh, sizeof(pppm_hit) * (size_t)n));
+    TRY_HIP(ctx, ctx->stage.copy_out(ctx->stream, hits, dh, sizeof(pppm_hit) * (size_t)n));
     return PPPM_OK;
 }
 
@@ -487,8 +457,8 @@ int pppm_hashgrid_build(void* ctx_raw, const float* pos, int64_t n, int32_t hash
     uint32_t* vals = build_grid(ctx, nullptr, ctx->scratch.as<float>(), nullptr, n, g, -1);
     TRY_HIP(ctx, hipGetLastError());
     std::vector<uint32_t> off((size_t)hash_size + 1);
-    if (n > 0 && sorted_idx) TRY_HIP(ctx, copy_to_host(ctx, ctx->stream, sorted_idx, vals, sizeof(uint32_t) * (size_t)n));
-    TRY_HIP(ctx, copy_to_host(ctx, ctx->stream, off.data(), ctx->off.p, sizeof(uint32_t) * off.size()));
+    if (n > 0 && sorted_idx) TRY_HIP(ctx, ctx->stage.copy_out(ctx->stream, sorted_idx, vals, sizeof(uint32_t) * (size_t)n));
+    TRY_HIP(ctx, ctx->stage.copy_out(ctx->stream, off.data(), ctx->off.p, sizeof(uint32_t) * off.size()));
     copy_ranges(off, hash_size, cell_start, cell_end);
     return PPPM_OK;
 }
@@ -591,7 +561,7 @@ int pppm_image_read(void* ctx_raw, double* rgb, int64_t n_values) {
     if (ctx->rp.method == PPPM_METHOD_HACHISUKA) {
         TRY_HIP(ctx, ctx->ppm_image.ensure(sizeof(double) * (size_t)nv));
         TRY_HIP(ctx, hachisuka_image(ctx, ctx->ppm_image.as<double>()));
-        TRY_HIP(ctx, copy_to_host(ctx, ctx->stream, rgb, ctx->ppm_image.p, sizeof(double) * (size_t)nv));
+        TRY_HIP(ctx, ctx->stage.copy_out(ctx->stream, rgb, ctx->ppm_image.p, sizeof(double) * (size_t)nv));
         return PPPM_OK;
     }
     TRY_HIP(ctx, hipStreamSynchronize(ctx->stream2));
@@ -601,7 +571,7 @@ int pppm_image_read(void* ctx_raw, double* rgb, int64_t n_values) {
     launch_image_average(ctx->stream, ctx->img_sum.as<float>(), ctx->img_comp.as<float>(), ctx->img_dsum.as<float>(),
                          ctx->img_dcomp.as<float>(), nv, inv, ctx->scratch.as<double>());
     TRY_HIP(ctx, hipGetLastError());
-    TRY_HIP(ctx, copy_to_host(ctx, ctx->stream, rgb, ctx->scratch.p, sizeof(double) * (size_t)nv));
+    TRY_HIP(ctx, ctx->stage.copy_out(ctx->stream, rgb, ctx->scratch.p, sizeof(double) * (size_t)nv));
     return PPPM_OK;
 }
 

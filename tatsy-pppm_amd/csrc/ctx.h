@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "stage.h"
 #include "traverse.h"
 
 namespace pppmi {
@@ -110,11 +111,8 @@ struct Ctx {
     // pinned host copies of the pipelined passes' counters, so that their
     // copy does not hold the host while the photon kernel runs
     HostCounters* pinned_counters = nullptr;
-    // two pinned buffers of STAGE_BYTES that copies to pageable host memory pass
-    // through (copy_to_host)
-    char* stage = nullptr;
-    hipEvent_t stage_ev[2] = {};
     int64_t pinned_count = 0;
+    HostStage stage;  // what results pass through on their way to the caller's memory
     hipEvent_t ev[13] = {};
     hipStream_t stream2 = nullptr;  // the eye pass runs here, concurrent with the photon pass
     hipStream_t stream3 = nullptr;  // the gather of pipelined passes (pppm_render_passes)
@@ -173,11 +171,6 @@ struct Ctx {
     void* noalloc_scratch = nullptr;
     hipError_t noalloc_err = hipSuccess;
 
-    ~Ctx() {
-        if (!stage) return;
-        (void)hipHostFree(stage);
-        for (auto& e : stage_ev) (void)hipEventDestroy(e);
-    }
     int fail(int code, const std::string& msg) {
         err = msg;
         return code;
@@ -250,7 +243,6 @@ uint32_t* build_grid(Ctx* c, const float4* pos4, const float* pos3, const uint32
 uint32_t* origin_order(Ctx* c, hipStream_t s, int64_t slots, int64_t n, const GridParams& g, const unsigned long long* slot_count,
                        bool starts_done = false);
 void origin_starts(Ctx* c, hipStream_t s);
-hipError_t copy_to_host(Ctx* c, hipStream_t s, void* dst, const void* src, size_t bytes);
 hipError_t ensure_sort_buffers(Ctx* c, int64_t n, uint32_t S);
 hipError_t ensure_hit_sort(Ctx* c, int64_t n);
 void sort_hitpoints(hipStream_t s, DBuf* hk, DBuf& hhist, const float4* hp, const float4* hw, int64_t cap,

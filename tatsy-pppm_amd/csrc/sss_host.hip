@@ -379,7 +379,7 @@ int pppm_dipole_eval(void* ctx_raw, const pppm_bsdf* material, const float* pts,
         }
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = copy_to_host(ctx, ctx->stream, out, dout, sizeof(float) * 3 * (size_t)n_query);
+    if (e == hipSuccess) e = ctx->stage.copy_out(ctx->stream, out, dout, sizeof(float) * 3 * (size_t)n_query);
     if (e != hipSuccess) return ctx->fail(PPPM_ERR_HIP, std::string("dipole: ") + hipGetErrorString(e));
     return PPPM_OK;
 }
