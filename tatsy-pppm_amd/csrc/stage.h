@@ -1,4 +1,4 @@
-// stage.h -- copies from the device to the caller's memory through pinned buffers.
+// stage.h -- copies from the device to the caller's memory.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -40,15 +40,28 @@ struct HostStage {
     }
 
     // Device memory src to dst, behind the work on s; complete on return, also
-    // where it fails (then no copy into the buffers is left on s).
+    // where it fails (then no copy is left on s).  Memory that the runtime knows
+    // (pinned, managed, a device's) takes one copy straight there.
     hipError_t copy_out(hipStream_t s, void* dst, const void* src, size_t bytes) {
-        hipError_t e = ready();
-        if (e != hipSuccess) return e;
+        hipError_t e;
+        if (known(dst)) {
+            if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+            return hipStreamSynchronize(s);
+        }
+        if ((e = ready()) != hipSuccess) return e;
         if ((e = staged(s, (char*)dst, (const char*)src, bytes)) != hipSuccess) (void)hipStreamSynchronize(s);
         return e;
     }
 
 private:
+    static bool known(const void* p) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();  // pageable memory is an error to some runtimes
+            return false;
+        }
+        return a.type != hipMemoryTypeUnregistered;
+    }
     hipError_t staged(hipStream_t s, char* dst, const char* src, size_t bytes) {
         hipError_t e;
         const size_t chunks = (bytes + STAGE_BYTES - 1) / STAGE_BYTES;

@@ -12,6 +12,8 @@
 static int calls, fail_at = -1;          // calls made, the one that fails
 static int buffers, events;              // alive
 static std::vector<std::function<void()>> queue;  // the stream's work not yet done
+static const char *pinned_lo, *pinned_hi;  // memory the runtime knows
+static int copies, last_error;
 static bool fails() { return calls++ == fail_at; }
 static void drain() {
     for (auto& f : queue) f();
@@ -55,8 +57,19 @@ hipError_t hipStreamSynchronize(hipStream_t) {
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     if (fails()) return hipErrorUnknown;
+    copies++;
     queue.push_back([=] { std::memcpy(d, s, n); });
     return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    if (p < pinned_lo || p >= pinned_hi) return (hipError_t)(last_error = hipErrorInvalidValue);
+    a->type = hipMemoryTypeHost;
+    return hipSuccess;
+}
+hipError_t hipGetLastError() {
+    const hipError_t e = (hipError_t)last_error;
+    last_error = hipSuccess;
+    return e;
 }
 }
 
@@ -91,6 +104,18 @@ int main() {
         expect(st.copy_out(nullptr, dst.data(), src.data(), src.size()) == hipSuccess, "works after a failure", at);
         expect(!std::memcmp(dst.data(), src.data(), src.size()), "with the right bytes", at);
     }
+    // pinned memory: one copy, straight there, no buffers made
+    pinned_lo = dst.data();
+    pinned_hi = pinned_lo + dst.size();
+    for (size_t n : {(size_t)1, STAGE_BYTES + 1, src.size()}) {
+        HostStage st;
+        copies = 0;
+        std::fill(dst.begin(), dst.end(), 0);
+        expect(st.copy_out(nullptr, dst.data(), src.data(), n) == hipSuccess, "copies to pinned memory", (long)n);
+        expect(!std::memcmp(dst.data(), src.data(), n) && queue.empty(), "the bytes arrive there", (long)n);
+        expect(copies == 1 && buffers == 0, "in one copy", copies);
+    }
+    expect(hipGetLastError() == hipSuccess, "no error is left behind", 0);
     expect(buffers == 0 && events == 0, "everything is given back", buffers + events);
     if (!failures) std::printf("OK\n");
     return failures != 0;
