@@ -34,7 +34,7 @@ hipError_t prepare_enqueued(Ctx* ctx) {
 // sentinel keys behind the records, and the pass index and radius come from
 // the device pass state (advanced first).  The image equals pppm_render_pass's
 // bit for bit for the same hash size.
-void enqueue_pass(Ctx* ctx, int photon_grid, int trace_keep) {
+void enqueue_pass(Ctx* ctx, int photon_grid, int trace_keep) {  // photon_grid <= ctx->photon_grid
     hipStream_t s = ctx->stream;
     PassDev* pd = ctx->pdev.as<PassDev>();
     Counters* dc = ctx->counters.as<Counters>();
@@ -225,7 +225,7 @@ int pppm_batch_add(void* batch, const float* tri_xyz, const int32_t* bsdf_id, in
     }
     BatchScene sc;
     sc.ctx = c;
-    sc.photon_grid = c->cu > 0 ? c->cu * PHOTON_BLOCKS_PER_CU : 2048;
+    sc.photon_grid = c->photon_grid;
     b->scenes.push_back(sc);
     b->drop_graph();
     if (index) *index = (int32_t)b->scenes.size() - 1;
@@ -249,6 +249,7 @@ int pppm_batch_tune(void* batch, int32_t tune_gather, int32_t tune_grid) {
         const int cu = c->cu > 0 ? c->cu : 256;
         if (tune_grid) grids = {cu, cu * 2, cu * 4, cu * 8};
         else grids = {sc.photon_grid};
+        c->photon_grid = *std::max_element(grids.begin(), grids.end());  // record slots for all of them
         double best = 1e30;
         int best_mode = base.gather_mode, best_grid = sc.photon_grid, best_keep = sc.trace_keep;
         // one timed pass per candidate after a warm-up pass; returns false on error
@@ -294,6 +295,7 @@ int pppm_batch_tune(void* batch, int32_t tune_gather, int32_t tune_grid) {
         }
         pppm_render_params p = base;
         p.gather_mode = best_mode;
+        c->photon_grid = best_grid;
         int rc = pppm_render_begin(c, &p);
         if (rc != PPPM_OK) return b->fail(rc, c->err);
         if (prepare_enqueued(c) != hipSuccess) return b->fail(PPPM_ERR_HIP, "tuning reset");

@@ -171,6 +171,7 @@ int pppm_create(void** out, int32_t device) {
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
         c->name = prop.gcnArchName;
         c->cu = prop.multiProcessorCount;
+        if (c->cu > 0) c->photon_grid = c->cu * PHOTON_BLOCKS_PER_CU;
         c->hbm = prop.totalGlobalMem;
     }
     c->noalloc_err = noalloc_setup(device, &c->noalloc_scratch);

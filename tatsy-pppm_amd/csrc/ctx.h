@@ -99,6 +99,7 @@ struct Ctx {
     // among its photon's records, records per photon, their exclusive scan
     DBuf rec_rank, rec_count, rec_start, rec_tiles;
     int64_t rec_slots = 0;  // record slots of ph_rec and rec_rank: cap and what chunks may leave empty
+    int photon_grid = 2048;  // blocks of the photon pass at most, which rec_slots is sized for
     // last pass
     bool last_valid = false;
     int64_t last_n = 0;

@@ -241,7 +241,7 @@ std::string hachisuka_pass(Ctx* c, pppm_pass_stats* st) {
     pa.count_traversal = c->count_traversal;
     pa.rec_rank = c->rec_rank.as<uint8_t>();
     pa.rec_count = c->rec_count.as<uint32_t>();
-    launch_photon_pass(s, pa, c->cu > 0 ? c->cu * PHOTON_BLOCKS_PER_CU : 2048);
+    launch_photon_pass(s, pa, c->photon_grid);
     HostCounters hcs;
     if (hipMemcpyAsync(&hcs, dc, sizeof(hcs), hipMemcpyDeviceToHost, s) != hipSuccess) return "count copy failed";
     if (hipStreamSynchronize(s) != hipSuccess) return std::string("pass: ") + hipGetErrorString(hipGetLastError());

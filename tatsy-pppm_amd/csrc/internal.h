@@ -175,16 +175,19 @@ __device__ inline int64_t hit_count(const Counters* c) {
 // pipelined passes of the caustic box in 79 ms against 75.
 #define PHOTON_WAVES 4
 #define PHOTON_BLOCKS_PER_CU PHOTON_WAVES
-// Record slots a photon-pass wave takes at a time: enough that it takes some
-// about once in ten shading rounds.
-#define RECORD_CHUNK 256
-// Blocks of the photon pass for a grid limit, and the record slots it may use
-// beyond the records it stores (two chunks begun per wave).
-inline int64_t photon_blocks(int64_t photons, int64_t grid_limit, int64_t lanes) {
-    return std::max<int64_t>(1, std::min(grid_limit, (photons + 4 * lanes - 1) / (4 * lanes)));
-}
-inline int64_t photon_spare_slots(int64_t photons, int cus) {  // for any grid up to 8 blocks per CU
-    return photon_blocks(photons, 8 * (int64_t)(cus > 0 ? cus : 256), 16) * 4 * 2 * RECORD_CHUNK;
+// Record slots a photon-pass wave takes at a time: RECORD_ROUNDS rounds in which
+// each of its paths stores one, so that it takes some about once in ten shading
+// rounds.
+#define RECORD_ROUNDS 4
+// Record slots that a pass may use beyond the records it stores, for any grid up
+// to grid_limit blocks of four waves: a wave of L paths ends with less than a
+// round's and a chunk's slots left over, (RECORD_ROUNDS + 1) L, and the waves
+// hold no more paths than fit the grid, nor than there are photons and one
+// block's ends (4 L - 1, L at most 64).  Sized for the most waves and the largest
+// chunk whatever the launch, a context took 139 MB for them from 131 k photons
+// on, now 22 MB there and 43 MB at most.
+inline int64_t photon_spare_slots(int64_t photons, int64_t grid_limit) {
+    return (RECORD_ROUNDS + 1) * std::min(photons + 255, 256 * grid_limit);
 }
 // rank of a record slot that holds no record
 #define NO_RECORD 255

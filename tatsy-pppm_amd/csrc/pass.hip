@@ -148,7 +148,7 @@ int pppm_render_begin(void* ctx_raw, const pppm_render_params* p) {
     TRY_HIP(ctx, hipMemcpy(ctx->lights.p, ld.data(), sizeof(LightDev) * (size_t)nl, hipMemcpyHostToDevice));
     const int64_t npix = (int64_t)ctx->cam.width * ctx->cam.height;
     const int64_t cap = ctx->cap;
-    ctx->rec_slots = cap + photon_spare_slots(p->photons, ctx->cu);
+    ctx->rec_slots = cap + photon_spare_slots(p->photons, ctx->photon_grid);
     TRY_HIP(ctx, ctx->ph_rec.ensure(sizeof(float4) * 2 * (size_t)ctx->rec_slots));
     TRY_HIP(ctx, ctx->rec_rank.ensure((size_t)ctx->rec_slots));
     TRY_HIP(ctx, ctx->rec_count.ensure(sizeof(uint32_t) * (size_t)p->photons));
@@ -209,7 +209,6 @@ int pppm_render_pass(void* ctx_raw, pppm_pass_stats* st) {
     const double radius = ctx->radii[(size_t)pass - 1];
     const int64_t npix = (int64_t)ctx->cam.width * ctx->cam.height;
     const int eye_grid = ctx->cu > 0 ? ctx->cu * EYE_BLOCKS_PER_CU : 2048;
-    const int photon_grid = ctx->cu > 0 ? ctx->cu * PHOTON_BLOCKS_PER_CU : 2048;
     Counters* dc = ctx->counters.as<Counters>();
     ctx->last_valid = false;
 
@@ -244,7 +243,7 @@ int pppm_render_pass(void* ctx_raw, pppm_pass_stats* st) {
     pa.count_traversal = ctx->count_traversal;
     pa.rec_rank = ctx->rec_rank.as<uint8_t>();
     pa.rec_count = ctx->rec_count.as<uint32_t>();
-    launch_photon_pass(s, pa, photon_grid);
+    launch_photon_pass(s, pa, ctx->photon_grid);
     TRY_HIP(ctx, hipGetLastError());
     TRY_HIP(ctx, hipEventRecord(ctx->ev[1], s));
     // the eye side is enqueued behind the photon kernel's launch: its fifteen
@@ -547,7 +546,6 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
     enum { ZERO, P0, P1, O0, ODONE, E0, E1, HDONE, G0, GEND, GDONE };
     const int NEV = 6;  // event ring: pass k records into pev[k % NEV]
     const int eye_grid = ctx->cu > 0 ? ctx->cu * EYE_BLOCKS_PER_CU : 2048;
-    const int photon_grid = ctx->cu > 0 ? ctx->cu * PHOTON_BLOCKS_PER_CU : 2048;
     const int32_t first = ctx->passes_done + 1;  // pass index of k = 0
     std::vector<float> times((size_t)count * 6, 0.0f);
     std::vector<int32_t> sizes((size_t)count, 0);
@@ -628,7 +626,7 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
         pa.count_traversal = ctx->count_traversal;
         pa.rec_rank = ctx->rec_rank.as<uint8_t>();
         pa.rec_count = ctx->rec_count.as<uint32_t>();
-        launch_photon_pass(A, pa, photon_grid);
+        launch_photon_pass(A, pa, ctx->photon_grid);
         TRY_HIP(ctx, hipGetLastError());
         TRY_HIP(ctx, hipEventRecord(E[P1], A));
         // the record starts per photon need only the photon kernel's counts;

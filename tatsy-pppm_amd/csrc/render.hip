@@ -153,14 +153,14 @@ struct WaveChunks {
     }
     // Before a shading round, by the whole wave: slots for all its lanes.
     __device__ inline void have_slots(const PhotonPassArgs& a) {
-        if (left < 64 && spare < 0) spare = take(&a.counters->record_slots, RECORD_CHUNK);
+        if (left < a.lanes && spare < 0) spare = take(&a.counters->record_slots, RECORD_ROUNDS * a.lanes);
     }
     // The slot of the k-th record of the round.
     __device__ inline int64_t slot(int k) const { return k < left ? cur + k : spare + (k - left); }
-    __device__ inline void used_slots(int k) {
+    __device__ inline void used_slots(const PhotonPassArgs& a, int k) {
         if (k > left) {
             cur = spare + (k - left);
-            left = RECORD_CHUNK - (k - left);
+            left = RECORD_ROUNDS * a.lanes - (k - left);
             spare = -1;
         } else {
             cur += k;
@@ -172,7 +172,7 @@ struct WaveChunks {
         const int lane = threadIdx.x & 63;
         for (int k = lane; k < left; k += 64)
             if (cur + k < a.slots) a.rec_rank[cur + k] = NO_RECORD;
-        for (int k = lane; spare >= 0 && k < RECORD_CHUNK; k += 64)
+        for (int k = lane; spare >= 0 && k < RECORD_ROUNDS * a.lanes; k += 64)
             if (spare + k < a.slots) a.rec_rank[spare + k] = NO_RECORD;
     }
 };
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PHOTON_WAVE
         {
             const int k = __popcll(__ballot(kept));
             n_stored += (unsigned long long)k;
-            ch.used_slots(k);
+            ch.used_slots(a, k);
         }
         const int paths = (int)__popcll(__ballot(live));
         if (paths == 0) {
@@ -672,7 +672,8 @@ void launch_photon_pass(hipStream_t s, const PhotonPassArgs& args, int grid_limi
     if (args.n_photons <= 0) return;
     PhotonPassArgs a = args;
     a.lanes = wave_ray_slots(a.n_photons, 4 * (int64_t)grid_limit);
-    const dim3 g((unsigned)photon_blocks(a.n_photons, grid_limit, a.lanes));
+    const int64_t blocks = (a.n_photons + 4 * a.lanes - 1) / (4 * a.lanes);
+    const dim3 g((unsigned)std::max<int64_t>(1, std::min<int64_t>(grid_limit, blocks)));
     const uint32_t lds = 4 * wave_rays_bytes(a.sc.stack);
     const bool env = a.sc.env != nullptr;
     if (a.count_traversal && env)

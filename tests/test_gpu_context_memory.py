@@ -1,0 +1,41 @@
+"""What a context takes of the device's memory, through the C ABI."""
+import ctypes as C
+
+import pytest
+
+import pppm_amd as P
+
+pytestmark = pytest.mark.gpu
+
+MiB = 1 << 20
+
+
+def _free():
+    hip = C.CDLL("/opt/rocm/lib/libamdhip64.so.7")  # already mapped: the library links it
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.fixture
+def ctx():
+    with P.Context(0) as c:
+        s = P.scenegen(P.SCENE_BOX, 1, 0, 16, 16)
+        c.upload(s)
+        c.build_bvh()
+        c.set_camera(s.camera)
+        yield c
+
+
+@pytest.mark.parametrize("photons", [2000, 131072, 1000000])
+def test_record_buffers(ctx, photons):
+    print(f"[case] {photons} photons", flush=True)
+    before = _free()
+    ctx.begin(photons, 1, 0.0866, capacity_factor=2.0)
+    used = before - _free()
+    # 102 bytes a record of the capacity, 8 a photon; 33 a slot that the photon
+    # pass may leave empty: five for each of at most 262,144 paths at a time
+    # (256 CUs of 16 waves of 64).  The rest, a few MiB of small buffers, each
+    # rounded up by the allocator
+    assert used <= (2 * 102 + 8) * photons + 33 * 5 * min(photons + 255, 262144) + 16 * MiB
+    assert ctx.render_pass()["photons_stored"] > 0
