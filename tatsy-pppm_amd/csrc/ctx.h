@@ -109,10 +109,9 @@ struct Ctx {
     uint32_t* last_sorted = nullptr;
     int32_t last_sub_bits = 0;  // the last pass ordered each bucket by a cell-local Morton code
     int32_t count_traversal = 0;  // passes run the node / triangle counting kernels
-    // pinned host copies of the pipelined passes' counters, so that their
-    // copy does not hold the host while the photon kernel runs
+    // pinned host copy of a pipelined pass's counters, so that the copy does
+    // not hold the host while the photon kernel runs
     HostCounters* pinned_counters = nullptr;
-    int64_t pinned_count = 0;
     HostStage stage;  // what results pass through on their way to the caller's memory
     hipEvent_t ev[13] = {};
     hipStream_t stream2 = nullptr;  // the eye pass runs here, concurrent with the photon pass

@@ -264,6 +264,8 @@ void launch_eye_pass(hipStream_t s, const EyePassArgs& a, int grid_limit);
 // img += the direct emission stored in the pixel slots without hit point
 // (an eye pass run with img_sum = null)
 void launch_direct_add(hipStream_t s, const float4* hp_w, int64_t np, float* img_sum, float* img_comp);
+// *out = the sum of a pass's counter copies
+void launch_counters_sum(hipStream_t s, const Counters* copies, Counters* out);
 // FP64 image average of n values
 void launch_image_average(hipStream_t s, const float* sum, const float* comp, const float* dsum, const float* dcomp,
                           int64_t n, double inv, double* out);

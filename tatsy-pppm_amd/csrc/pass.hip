@@ -530,15 +530,9 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
     }
     for (int i = 0; i < 4; i++) TRY_HIP(ctx, ctx->hk_alt[i].ensure(ctx->hk[i].n));
     TRY_HIP(ctx, ctx->hhist_alt.ensure(ctx->hhist.n));
-    TRY_HIP(ctx, ctx->pass_counters.ensure(sizeof(HostCounters) * (size_t)count));
-    if (ctx->pinned_count < count) {
-        (void)hipHostFree(ctx->pinned_counters);
-        ctx->pinned_counters = nullptr;
-        ctx->pinned_count = 0;
-        TRY_HIP(ctx, hipHostMalloc((void**)&ctx->pinned_counters, sizeof(HostCounters) * (size_t)count,
-                                   hipHostMallocDefault));
-        ctx->pinned_count = count;
-    }
+    TRY_HIP(ctx, ctx->pass_counters.ensure(sizeof(Counters) * (size_t)count));
+    if (!ctx->pinned_counters)
+        TRY_HIP(ctx, hipHostMalloc((void**)&ctx->pinned_counters, sizeof(HostCounters), hipHostMallocDefault));
     hipStream_t A = ctx->stream, Cs = ctx->stream3;
     hipStream_t Bq[2] = {ctx->stream2, ctx->stream4};
     DBuf* hkq[2] = {ctx->hk, ctx->hk_alt};
@@ -635,13 +629,13 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
         // photons run (its event set was last used by pass k - 4, whose times
         // were read in the last iteration)
         origin_starts(ctx, A);
-        TRY_HIP(ctx, hipMemcpyAsync(&ctx->pinned_counters[k], dc, sizeof(HostCounters), hipMemcpyDeviceToHost, A));
+        TRY_HIP(ctx, hipMemcpyAsync(ctx->pinned_counters, dc, sizeof(HostCounters), hipMemcpyDeviceToHost, A));
         if (k >= 3) read_times(k - 3);
         if (k + 2 < count) TRY_HIP(ctx, enqueue_eye(k + 2));
         // the stored count sizes the sorts; meanwhile the eye passes and the
         // previous gather run
         TRY_HIP(ctx, hipStreamSynchronize(A));
-        const Counters hc = ctx->pinned_counters[k].sum();
+        const Counters hc = ctx->pinned_counters->sum();
         const int64_t n = (int64_t)hc.photons_stored;
         if (n > ctx->cap) {
             (void)hipDeviceSynchronize();
@@ -695,8 +689,8 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
         launch_gather(Cs, ga);
         TRY_HIP(ctx, hipGetLastError());
         TRY_HIP(ctx, hipEventRecord(E[GEND], Cs));
-        TRY_HIP(ctx, hipMemcpyAsync(ctx->pass_counters.as<HostCounters>() + k, dc, sizeof(HostCounters),
-                                    hipMemcpyDeviceToDevice, Cs));
+        launch_counters_sum(Cs, dc, ctx->pass_counters.as<Counters>() + k);
+        TRY_HIP(ctx, hipGetLastError());
         TRY_HIP(ctx, hipEventRecord(E[GDONE], Cs));
         ctx->passes_done = pass;
         ctx->last_n = n;
@@ -729,11 +723,8 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
         swap_buf(set[0].hp_w_s, set[last].hp_w_s);
         swap_buf(set[0].counters, set[last].counters);
     }
-    std::vector<HostCounters> copies((size_t)count);
-    TRY_HIP(ctx, hipMemcpy(copies.data(), ctx->pass_counters.p, sizeof(HostCounters) * (size_t)count,
-                           hipMemcpyDeviceToHost));
     std::vector<Counters> dcs((size_t)count);
-    for (int32_t k = 0; k < count; k++) dcs[(size_t)k] = copies[(size_t)k].sum();
+    TRY_HIP(ctx, hipMemcpy(dcs.data(), ctx->pass_counters.p, sizeof(Counters) * (size_t)count, hipMemcpyDeviceToHost));
     ctx->last_valid = true;
     if (stats) {
         for (int32_t k = 0; k < count; k++) {

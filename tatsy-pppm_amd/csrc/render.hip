@@ -631,6 +631,17 @@ __global__ void k_capacity_check(PassDev* pd, const Counters* c, int64_t cap) {
     if ((int64_t)stored > cap || (int64_t)c->irr_stored > cap) pd->overflow = 1u;
 }
 
+// One thread per word of the counters.
+__global__ void k_counters_sum(const Counters* __restrict__ copies, Counters* __restrict__ out) {
+    constexpr int WORDS = sizeof(Counters) / sizeof(unsigned long long);
+    static_assert(WORDS <= 64, "one wave sums them");
+    if (threadIdx.x >= WORDS) return;
+    const unsigned long long* c = reinterpret_cast<const unsigned long long*>(copies) + threadIdx.x;
+    unsigned long long sum = 0;
+    for (int k = 0; k < COUNTER_COPIES; k++) sum += c[k * WORDS];
+    reinterpret_cast<unsigned long long*>(out)[threadIdx.x] = sum;
+}
+
 __global__ void k_permute2(const float4* __restrict__ a_in, const float4* __restrict__ b_in,
                            const uint32_t* __restrict__ perm, const uint32_t* __restrict__ perm2,
                            int64_t n, float4* __restrict__ a_out, float4* __restrict__ b_out, int stride) {
@@ -715,6 +726,10 @@ void launch_image_encode(hipStream_t s, const float* sum, const float* comp, con
     if (npix <= 0) return;
     hipLaunchKernelGGL(k_image_encode, dim3(grid1(npix, 256)), dim3(256), 0, s, sum, comp, dsum, dcomp, npix, inv, fmt,
                        ginv, out8, outf);
+}
+
+void launch_counters_sum(hipStream_t s, const Counters* copies, Counters* out) {
+    hipLaunchKernelGGL(k_counters_sum, dim3(1), dim3(64), 0, s, copies, out);
 }
 
 void launch_image_average(hipStream_t s, const float* sum, const float* comp, const float* dsum, const float* dcomp,

@@ -39,3 +39,19 @@ def test_record_buffers(ctx, photons):
     # rounded up by the allocator
     assert used <= (2 * 102 + 8) * photons + 33 * 5 * min(photons + 255, 262144) + 16 * MiB
     assert ctx.render_pass()["photons_stored"] > 0
+
+
+def test_counters_of_many_pipelined_passes(ctx):
+    # one line of 256 bytes a pass, whatever the copies that its kernels add to
+    passes = 4096
+    ctx.begin(100, passes + 4, 0.0866)
+    ctx.render_passes(4)
+    before = _free()
+    st = ctx.render_passes(passes)
+    assert before - _free() <= 256 * passes + 4 * MiB
+    assert len(st) == passes and st[-1]["pass_index"] == passes + 4
+    # the counts are those of single passes
+    ctx.begin(100, 6, 0.0866)
+    single = [ctx.render_pass() for _ in range(6)]
+    for k in ("photons_stored", "photon_segments", "eye_segments", "hitpoints", "gather_candidates", "gather_inradius"):
+        assert [s[k] for s in single[4:]] == [s[k] for s in st[:2]], k
