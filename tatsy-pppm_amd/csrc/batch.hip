@@ -75,8 +75,7 @@ void enqueue_pass(Ctx* ctx, int photon_grid, int trace_keep) {  // photon_grid <
     g.pd = pd;
     const int keep = 4;
     const uint32_t* perm1 = origin_order(ctx, s, ctx->rec_slots, cap, g, &dc->record_slots);
-    const uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, cap, g, keep,
-                                        &dc->record_slots, nullptr, true);
+    const uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, cap, g, keep, GRID_KEYS_SENTINELS);
     launch_gather_layout(s, ctx->ph_rec.as<float4>(), ctx->ph_rec.as<float4>() + 1, nullptr, sorted, cap,
                          ctx->ph_a.as<float4>(), ctx->ph_b.as<float4>(),
                          gather_compact(ctx->rp.gather_mode) ? nullptr : ctx->ph_c.as<float4>(),

@@ -60,13 +60,8 @@ void cross3(const double a[3], const double b[3], double o[3]) {
     o[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-// Builds the grid (sort by bucket of (pos4 or pos3) through perm) into the
-// context's sort buffers, avoiding the buffer `keep` (index into u[], or -1).
-// Returns the buffer holding the sorted values (grid sorted_idx).
-// With a device count the n slots hold *count records followed by unused
-// ones, whose keys sort behind every bucket.
-// Bits of a bucket id in the grid sort key (with a device count, one more
-// value for the sentinel of unused slots).
+// Bits of a bucket id in the grid sort key (where unused slots have a sentinel
+// for a key, one more value).
 int grid_bucket_bits(uint32_t size, bool sentinel) {
     return sentinel ? bits_for((uint64_t)size) : bits_for(size > 0 ? (uint64_t)(size - 1) : 0);
 }
@@ -82,18 +77,18 @@ int render_sub_bits(const Ctx* c, uint32_t size) {
     return std::max(0, std::min(3, (32 - grid_bucket_bits(size, true)) / 3));
 }
 
+// Builds the grid (sort by bucket of (pos4 or pos3) through perm) into the
+// context's sort buffers, avoiding the buffer `keep` (index into u[], or -1).
+// Returns the buffer holding the sorted values (grid sorted_idx).
 uint32_t* build_grid(Ctx* c, const float4* pos4, const float* pos3, const uint32_t* perm, int64_t n,
-                     const GridParams& g, int keep, const unsigned long long* count, uint32_t* off_out,
-                     bool keys_ready) {
+                     const GridParams& g, int keep, GridKeys how, uint32_t* off_out) {
     uint32_t* b[4];
     int k = 0;
     for (int i = 0; i < 5 && k < 4; i++)
         if (i != keep) b[k++] = c->u[i].as<uint32_t>();
-    const int bucket_bits = grid_bucket_bits(g.size, count != nullptr);
     const int shift = 3 * g.sub_bits;
-    const int bits = bucket_bits + shift;
-    const uint32_t sentinel = bits >= 32 ? 0xFFFFFFFFu : (uint32_t)((1ull << bits) - 1);
-    if (!keys_ready) launch_point_keys(c->stream, pos4, pos3, perm, n, g, b[0], b[1], count, sentinel);
+    const int bits = grid_bucket_bits(g.size, how == GRID_KEYS_SENTINELS) + shift;
+    if (how == GRID_KEYS_MAKE) launch_point_keys(c->stream, pos4, pos3, perm, n, g, b[0], b[1]);
     bool alt = radix_sort_pairs(c->stream, b[0], b[1], b[2], b[3], c->hist.as<uint32_t>(), n, bits);
     uint32_t* keys = alt ? b[2] : b[0];
     uint32_t* vals = alt ? b[3] : b[1];
@@ -106,7 +101,8 @@ uint32_t* build_grid(Ctx* c, const float4* pos4, const float* pos3, const uint32
 // The photon records of a pass in origin order (stable by photon index) with
 // their grid keys, from the ranks and counts the photon pass wrote: perm1
 // (origin position -> record slot) in u[4], keys and values (record slots) in
-// u[0], u[1] for build_grid(..., keep = 4, keys_ready).  Returns perm1.
+// u[0], u[1] for build_grid(..., keep = 4, GRID_KEYS_READY, or GRID_KEYS_SENTINELS
+// with a slot count).  Returns perm1.
 void origin_starts(Ctx* c, hipStream_t s) {
     launch_origin_starts(s, c->rec_count.as<uint32_t>(), c->rp.photons, c->rec_tiles.as<uint32_t>(),
                          c->rec_start.as<uint32_t>());

@@ -231,12 +231,12 @@ int grid_bucket_bits(uint32_t size, bool sentinel);
 int render_sub_bits(const Ctx* c, uint32_t size);
 // Builds the grid (sort by bucket of (pos4 or pos3) through perm) into the
 // context's sort buffers, avoiding the buffer `keep` (index into u[], or -1).
-// Returns the buffer holding the sorted values (grid sorted_idx).  With a
-// device count the n slots hold *count records followed by unused ones, whose
-// keys sort behind every bucket.
+// Returns the buffer holding the sorted values (grid sorted_idx).
+// Where the n keys come from: made here, in u[0] and u[1] already, or there
+// with a sentinel, behind every bucket, in each position that holds no record.
+enum GridKeys { GRID_KEYS_MAKE, GRID_KEYS_READY, GRID_KEYS_SENTINELS };
 uint32_t* build_grid(Ctx* c, const float4* pos4, const float* pos3, const uint32_t* perm, int64_t n,
-                     const GridParams& g, int keep, const unsigned long long* count = nullptr,
-                     uint32_t* off_out = nullptr, bool keys_ready = false);
+                     const GridParams& g, int keep, GridKeys how = GRID_KEYS_MAKE, uint32_t* off_out = nullptr);
 // The photon records in origin order (photon index, then rank); with
 // starts_done the per-photon record starts (origin_starts, which needs only
 // the photon pass's per-photon counts) are already enqueued on s.

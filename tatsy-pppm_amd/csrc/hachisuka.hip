@@ -279,7 +279,7 @@ std::string hachisuka_pass(Ctx* c, pppm_pass_stats* st) {
     g.sub_bits = 0;
     if (c->off.ensure(sizeof(uint32_t) * ((size_t)S + 1)) != hipSuccess) return "offset buffer allocation failed";
     uint32_t* perm1 = origin_order(c, s, std::min((int64_t)hc.record_slots, c->rec_slots), n, g, nullptr);
-    uint32_t* sorted = build_grid(c, nullptr, nullptr, perm1, n, g, 4, nullptr, nullptr, true);
+    uint32_t* sorted = build_grid(c, nullptr, nullptr, perm1, n, g, 4, GRID_KEYS_READY);
     launch_gather_layout(s, c->ph_rec.as<float4>(), c->ph_rec.as<float4>() + 1, nullptr, sorted, n,
                          c->ph_a.as<float4>(), c->ph_b.as<float4>(), nullptr, nullptr, 2);
     PpmArgs u;

@@ -54,15 +54,9 @@ __device__ inline uint32_t point_key(double x, double y, double z, const GridPar
 
 __global__ void k_point_keys(const float4* __restrict__ pos4, const float* __restrict__ pos3,
                              const uint32_t* __restrict__ perm, int64_t n, GridParams g,
-                             uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                             const unsigned long long* __restrict__ count, uint32_t sentinel) {
+                             uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    if (count && i >= (int64_t)min((unsigned long long)n, *count)) {
-        keys[i] = sentinel;
-        vals[i] = (uint32_t)i;
-        return;
-    }
     int64_t j = perm ? (int64_t)perm[i] : i;
     double x, y, z;
     if (pos4) {
@@ -364,11 +358,10 @@ __global__ void k_scan_u64_add(uint64_t* data, int64_t n, const uint64_t* block_
 static inline unsigned grid1(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 void launch_point_keys(hipStream_t s, const float4* pos4, const float* pos3, const uint32_t* perm,
-                       int64_t n, GridParams g, uint32_t* keys, uint32_t* vals, const unsigned long long* count,
-                       uint32_t sentinel) {
+                       int64_t n, GridParams g, uint32_t* keys, uint32_t* vals) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_point_keys, dim3(grid1(n, 256)), dim3(256), 0, s, pos4, pos3, perm, n, g,
-                       keys, vals, count, sentinel);
+                       keys, vals);
 }
 
 int64_t origin_tiles(int64_t photons) { return (photons + ORIGIN_TILE - 1) / ORIGIN_TILE; }

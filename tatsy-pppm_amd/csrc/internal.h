@@ -61,11 +61,9 @@ struct GridParams {
     const PassDev* pd = nullptr;  // when set, the scale is read from it
 };
 __device__ __forceinline__ double grid_scale(const GridParams& g) { return g.pd ? g.pd->scale : g.scale; }
-// keys[i] = hash(cell(pos[perm ? perm[i] : i])), vals[i] = i; with a device
-// count, slots i >= min(*count, n) get key `sentinel` (>= size)
+// keys[i] = hash(cell(pos[perm ? perm[i] : i])), vals[i] = i
 void launch_point_keys(hipStream_t s, const float4* pos4, const float* pos3, const uint32_t* perm,
-                       int64_t n, GridParams g, uint32_t* keys, uint32_t* vals,
-                       const unsigned long long* count = nullptr, uint32_t sentinel = 0xFFFFFFFFu);
+                       int64_t n, GridParams g, uint32_t* keys, uint32_t* vals);
 // Origin order without a sort (see k_origin_point_keys): start[i] = number of
 // records of photons 0..i-1, from the per-photon counts the photon pass wrote
 // (tile_sums: origin_tiles(photons) words of scratch) ...

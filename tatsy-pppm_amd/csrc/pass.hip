@@ -300,7 +300,7 @@ int pppm_render_pass(void* ctx_raw, pppm_pass_stats* st) {
     const int keep = 4;
     uint32_t* perm1 = origin_order(ctx, s, std::min((int64_t)hc.record_slots, ctx->rec_slots), n, g, nullptr);
     TRY_HIP(ctx, hipEventRecord(ctx->ev[2], s));
-    uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, n, g, keep, nullptr, nullptr, true);
+    uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, n, g, keep, GRID_KEYS_READY);
     launch_gather_layout(s, ctx->ph_rec.as<float4>(), ctx->ph_rec.as<float4>() + 1, nullptr, sorted, n,
                          ctx->ph_a.as<float4>(), ctx->ph_b.as<float4>(),
                          gather_compact(ctx->rp.gather_mode) ? nullptr : ctx->ph_c.as<float4>(),
@@ -654,8 +654,8 @@ int pppm_render_passes(void* ctx_raw, int32_t count, pppm_pass_stats* stats) {
         const int keep = 4;
         uint32_t* perm1 = origin_order(ctx, A, std::min((int64_t)hc.record_slots, ctx->rec_slots), n, g, nullptr, true);
         ctx->stream = A;
-        uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, n, g, keep, nullptr,
-                                      S.off->as<uint32_t>(), true);
+        uint32_t* sorted = build_grid(ctx, nullptr, nullptr, perm1, n, g, keep, GRID_KEYS_READY,
+                                      S.off->as<uint32_t>());
         ctx->stream = keep_stream;
         launch_gather_layout(A, ctx->ph_rec.as<float4>(), ctx->ph_rec.as<float4>() + 1, nullptr, sorted, n,
                              S.ph_a->as<float4>(), S.ph_b->as<float4>(),
