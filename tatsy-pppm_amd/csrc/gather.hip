@@ -11,11 +11,13 @@
 // (Phi, key), with a box per 32-record block; for the others three 16-byte
 // words (x, y, z, n_x) (n_y, n_z, Phi_r, Phi_g) (Phi_b, key, -, -) with the
 // normal decoded once.  Hit points arrive sorted along a Morton curve of half
-// cells (edge r), so neighbouring lanes share their eight buckets.  Four
+// cells (edge r), so neighbouring lanes share their eight buckets.  Five
 // kernels compute the same sum:
 //   k_gather_lanes (default): eight lanes per hit point walking its own buckets;
 //     inside a bucket the records follow a cell-local Morton order and blocks
 //     of 32 records whose bounding box misses the ball are skipped.
+//   k_gather_ordered: one lane per hit point, the same records summed one after
+//     the other (the irradiance points of a translucent object).
 //   k_gather_blocks: a wave walks the union of its lanes' buckets block by
 //     block, skips the blocks no lane needs (the lanes kernel's decisions) and
 //     stages the others in LDS for all 64 lanes.

@@ -168,9 +168,9 @@ __device__ inline int64_t hit_count(const Counters* c) {
 
 // Waves per SIMD of the photon kernel, which its registers are held to, and so
 // its persistent blocks of four waves per CU (every wave starts on photons of
-// its own).  Four take 98 registers and leave room for a wave of the gather on
-// the same SIMD; five (96, two spilled) trace a pass alone as fast and eight
-// pipelined passes of the caustic box in 79 ms against 75.
+// its own).  Four take 96 registers and leave room for a wave of the gather on
+// the same SIMD; five trace a pass alone as fast and eight pipelined passes of
+// the caustic box 5 % slower (79 ms against 75 when that was measured).
 #define PHOTON_WAVES 4
 #define PHOTON_BLOCKS_PER_CU PHOTON_WAVES
 // Record slots a photon-pass wave takes at a time: RECORD_ROUNDS rounds in which

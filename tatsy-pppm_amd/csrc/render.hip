@@ -11,7 +11,6 @@
 
 namespace {
 
-
 // Append one record per active lane with one atomic per wave; returns the slot.
 __device__ inline unsigned long long wave_append(unsigned long long* counter) {
     const uint64_t m = __ballot(1);
@@ -22,7 +21,6 @@ __device__ inline unsigned long long wave_append(unsigned long long* counter) {
     base = __shfl(base, leader);
     return base + (unsigned long long)__popcll(m & lanemask_lt());
 }
-
 
 // sampler.cc:17-32 (cosine-weighted direction about w)
 __device__ inline v3f on_hemisphere(v3f w, float r1, float r2) {

@@ -10,9 +10,9 @@
 // rays of a wave, the latency of the chain of node fetches: with one ray per
 // lane the four slab tests and the sort ran in every lane with 13 of 64 lanes
 // busy on average; here a step is half as long and the lanes it occupies do
-// work.  Photon pass of the caustic box (0.7 M triangles, 8.9 M rays): 4.2 ms
-// with one ray per lane, 3.4 ms with a quad per ray; 0.91 -> 0.83 ms on 60 k
-// triangles, 0.38 -> 0.33 ms at 200 k photons, 0.20 -> 0.12 ms at 10 k.  What
+// work.  Photon pass of the caustic box (0.7 M triangles, 8.9 M rays), a pass by
+// itself: 4.2 ms with one ray per lane, 3.1 ms with a quad per ray; 0.91 -> 0.77 ms
+// on 60 k triangles, 0.38 -> 0.26 ms at 200 k photons, 0.30 -> 0.16 ms at 10 k.  What
 // is left is the latency of node fetches: a step waits for the slowest of up to
 // sixteen, and four in ten miss the 4 MiB L2 of their die.
 // The loop is the while-while form with postponed leaves of Aila and Laine
@@ -195,9 +195,9 @@ __device__ inline void rays_trace(const SceneDev& sc, const WaveRays& w, QuadRay
             q.cur = POP();
         }
         // inner nodes, until the quads with a leaf waiting are more than twice
-        // those that still look for one (photon pass 3.2 ms; 3.7 ms waiting for
-        // the last quad, 3.3 and 3.4 ms at once and five times; with few rays
-        // the ratio does not matter)
+        // those that still look for one (a photon pass takes 16 % longer waiting
+        // for the last quad, 3 and 6 % at once and five times; with few rays the
+        // ratio does not matter)
         while (true) {
             const bool inner = (uint32_t)q.cur < (uint32_t)EMPTY_REF;
             const int stepping = (int)__popcll(__ballot(inner && leaf >= 0));

@@ -3,7 +3,7 @@ through the C ABI.
 
 A ray's hit does not depend on the rays traced beside it, so the first n rays
 of a batch alone hit what they hit in the whole batch, bit for bit; the whole
-batch, rays with an interval of their own, leaves of one to four triangles and
+batch, rays with an interval of their own, leaves of one and two triangles and
 eye passes of odd sizes are held against the oracle.
 """
 import numpy as np
